@@ -705,3 +705,25 @@ def test_decode_overflow_stays_infinite(device):
     assert torch.equal(torch.isposinf(out), torch.isposinf(want)) and not out.isnan().any()
     assert torch.isposinf(out[1::2]).all() and torch.isfinite(out[::2]).all()
     assert_close(host_bits(out[::2].contiguous()), host_bits(want[::2].contiguous()), "finite tokens", cos_tol=0.99999)
+
+
+def test_decode_stage_b_adds_waves_in_double(device):
+    """Stage B's waves take 256 k each: sums of 2^24, 1 and -2^24 from three of
+    them have to give the 1, which fp32 sums in wave order lose."""
+    T, E, K, H, O = 64, 2, 2048, 2048, 4096
+    announce(f"decode stage B sums of the waves T={T} H={H} O={O}")
+    W1 = np.zeros((E, H, K // 2), np.uint8)
+    W1[..., 0] = 0x02                              # W1 x = x[0] = 128, and so is its silu
+    W2 = np.zeros((E, O, H // 2), np.uint8)
+    x = np.zeros((T, K), np.float32)
+    x[:, 0] = 128.0
+    for i, v in ((1, 2.0 ** 17), (257, 2.0 ** -7), (513, -2.0 ** 17)):
+        W2[..., i // 2] = 0x20
+        x[:, i] = v                                # M[i] = 128 x[i]
+    mats = [{"packed": dev_u8(W1, device), "scale": dev_u8(np.full((E, H, K // 32), 127), device)},
+            _one_hot_rows(E, H, K, device),
+            {"packed": dev_u8(W2, device), "scale": dev_u8(np.full((E, O, H // 32), 127), device)}]
+    ids = torch.zeros((T, 1), dtype=torch.int32, device=device)
+    xd = torch.from_numpy(x).to(torch.bfloat16).to(device)
+    out = gb.mxfp4_moe_grouped_gemv(xd, *mats, ids, torch.ones((T, 1), device=device))
+    assert torch.equal(out, torch.ones_like(out))
