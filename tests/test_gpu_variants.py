@@ -727,3 +727,35 @@ def test_decode_stage_b_adds_waves_in_double(device):
     xd = torch.from_numpy(x).to(torch.bfloat16).to(device)
     out = gb.mxfp4_moe_grouped_gemv(xd, *mats, ids, torch.ones((T, 1), device=device))
     assert torch.equal(out, torch.ones_like(out))
+
+
+@pytest.mark.parametrize("K,H", [(1024, 2048), (2048, 1024), (4096, 2048), (3072, 1280)])
+@pytest.mark.parametrize("small", [0, 1, 2])
+def test_decode_batches_smallest_scales(device, small, K, H):
+    """All scale bytes of one matrix 0 or 1 (2^-127, 2^-126), with activations or
+    other scales that make the result an ordinary number: the weights are exact
+    on the matrix cores too, so the general kernels give it up to the rounding of
+    sums and M. One expert of W2 has no such byte."""
+    T, topk, E, O = 33, 8, 16, 192
+    announce(f"decode batches smallest scales K={K} H={H} matrix {small}")
+    rng = np.random.default_rng(9750 + K)
+    mats = []
+    for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
+        p, s = synth.mxfp4_weight(9760 + 2 * m, rows, cols, E)
+        if m == small:
+            s = rng.integers(0, 2, s.shape).astype(np.uint8)
+            if m == 2:
+                s[3] = rng.integers(2, 4, s[3].shape)
+        elif m == 1 and small == 2:
+            s = (s + 100).astype(np.uint8)         # M about 2^100
+        mats.append({"packed": dev_u8(p, device), "scale": dev_u8(s, device)})
+    scale = 1.0 if small == 2 else 2.0 ** 100      # the other of W1 x and W3 x about 2^100
+    x = mx.bf16_round(mx.bf16_to_f32(synth.normal_bf16(9770, (T, K))) * np.float32(scale))
+    ids = np.stack([rng.permutation(E)[:topk] for _ in range(T)]).astype(np.int32)
+    w = (rng.random((T, topk)) + 0.1).astype(np.float32)
+    args = torch.from_numpy(ids).to(device), dev_f32(w, device)
+    gen = [{"packed": m["packed"], "scale": _at_offset(m["scale"], 1)} for m in mats]
+    out = gb.mxfp4_moe_grouped_gemv(dev_bf16(x, device), *mats, *args)
+    want = host_bits(gb.mxfp4_moe_grouped_gemv(dev_bf16(x, device), *gen, *args))
+    assert np.median(np.abs(mx.bf16_to_f32(want))) > 2.0 ** -100
+    assert_close(host_bits(out), want, "smallest scales", cos_tol=0.99999)
