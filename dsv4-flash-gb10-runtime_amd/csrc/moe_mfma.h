@@ -37,3 +37,8 @@ hipError_t mfma_down(const uint16_t* M, const uint8_t* w2, const uint8_t* s2, in
                      const SlotTables& st, uint16_t* out, hipStream_t stream);
 
 }  // namespace dsv4
+
+// Which stages of a decode batch with 16-byte aligned operands run on the
+// matrix cores: bit 0 stage A, bit 1 stage B (so that the tests can name the
+// path that a case takes; needs no GPU).
+extern "C" int mxfp4_moe_decode_stages(int T, int topk, int n_experts, int K_in, int hidden, int out_dim);

@@ -1890,25 +1890,33 @@ int launch_route(const float* logits, const int32_t* ids, const float* weights, 
 // one token never does: its GEMV kernels are the faster ones and gate in their
 // first launch). Where most experts serve one or two tokens the GEMV kernels
 // are at the weight stream's rate; with more, their dots per token bound them.
-// Measured in us for the layer, GEMV / that stage alone on MFMA (MI355X):
-//   A, K = 4096, P pairs and E experts: P / E = 1 204 / 217, 388 / 403 and
-//     110 / 118; 1.5 148 / 148, 274 / 268, 532 / 515; 1.75 161 / 154; 2 181 /
-//     162, 338 / 311, 663 / 598, with 8 experts 36 / 32; K = 2048: 1.5 68 / 71,
-//     2 83 / 80 and 50 / 47. K between (its lanes past the row idle in the GEMV):
-//     K = 3072 at 0.06 43.9 / 42.3, 0.25 144 / 138, 1 125 / 107; 2560 at 0.5
-//     125 / 121; 3584 at 1 256 / 209; but K = 1536 at 1 91 / 96.
+// Measured in us per stage, MFMA / GEMV, P pairs and E experts, every call on
+// weights of its own (MI355X).
+//   A, K = 4096: P / E = 1 282 / 251 and 79 / 68, 1.5 341 / 346 and 97 / 93, 1.75
+//     359 / 387 and 99 / 102, 2 376 / 429, 3 112 / 154; K = 2048: 1 80 / 72 and 27 /
+//     25, 1.5 93 / 99 and 32 / 32, 1.75 33 / 35, 2 101 / 127. Few pairs are one
+//     short round of workgroups that waits for its first loads: 8 of 4096 x 2048
+//     18.6 / 13.5, 16 20.5 / 21.7 and 20.1 / 22.2, 48 of 4096 x 512 17.8 / 15.4, 64
+//     20.2 / 24.2; 16 of 2048 x 1024 11.8 / 9.6, 28 13.2 / 12.9, 32 13.5 / 14.4.
+//     K between, where lanes past the row idle in the GEMV: K = 3072 8 pairs
+//     17.4 / 17.0, 16 26.3 / 28.8, 32 47.9 / 53.8, P / E = 1 227 / 308; 2560 (hidden
+//     1536) 16 pairs 21.3 / 19.5, 24 30.7 / 27.2, 32 32.7 / 32.9, 64 58.6 / 61.0,
+//     P / E = 1 144 / 197; 3584 (1408) 24 38.8 / 35.0, 32 40.6 / 44.3.
 //   B, hidden = 2048: 1 204 / 214, 1.5 274 / 272 and 148 / 149, 1.75 161 / 157,
 //     2 181 / 175, 338 / 320, 663 / 627; hidden = 1536: 0.75 145.6 / 146.4, 1.12
 //     193 / 183 and 369 / 349; 1024: 0.5 98 / 89 and 34 / 37, 1 53.2 / 52.6 and
 //     165 / 143. Few pairs leave too few slots for its ring: 16 pairs 38 / 42, 32
 //     61.9 / 62.0, 31.7 / 32.0 and 38 / 41, 48 71 / 64, 64 99 / 96.
-bool mfma_stage_a(int T, int K, const ExpertSet& es) {
-    return T > 1 && ((K > 2048 && K < 4096) || 4 * es.n_pairs >= 7 * es.n_experts);
+bool mfma_stage_a(int T, int K, int hidden, int n_pairs, int n_experts) {
+    const int work = n_pairs * hidden;            // at most 1024 * 4096
+    if (T < 2) return false;
+    if (4 * n_pairs >= 7 * n_experts) return work >= 16 * 2048;
+    return K > 2048 && K < 4096 && work >= 32 * 1536;
 }
 
-bool mfma_stage_b(int T, int hidden, const ExpertSet& es) {
-    return T > 1 && es.n_pairs >= 48 &&
-           (hidden < 2048 ? es.n_pairs >= es.n_experts : 4 * es.n_pairs >= 7 * es.n_experts);
+bool mfma_stage_b(int T, int hidden, int n_pairs, int n_experts) {
+    return T > 1 && n_pairs >= 48 &&
+           (hidden < 2048 ? n_pairs >= n_experts : 4 * n_pairs >= 7 * n_experts);
 }
 
 SlotTables slot_tables(const ExpertSet& es) {
@@ -1932,7 +1940,8 @@ int launch_swiglu(const dsv4_bf16_t* x, const uint8_t* W1_packed, const uint8_t*
     A.es = c.es;
     const bool al = aligned16(x) && aligned16(W1_packed) && aligned16(W3_packed);
     hipError_t e;
-    if (mfma_stage_a(T, K_in, c.es) && mfma_swiglu_ok(K_in, hidden, x, W1_packed, W3_packed, W1_scale, W3_scale)) {
+    if (mfma_stage_a(T, K_in, hidden, c.es.n_pairs, c.es.n_experts) &&
+        mfma_swiglu_ok(K_in, hidden, x, W1_packed, W3_packed, W1_scale, W3_scale)) {
         e = mfma_swiglu(A.x, W1_packed, W3_packed, W1_scale, W3_scale, T, K_in, hidden, slot_tables(c.es), c.M, stream);
     } else if (gate != nullptr) {
         A.gate = *gate;
@@ -1965,7 +1974,8 @@ int launch_down(const uint8_t* W2_packed, const uint8_t* W2_scale, int T, int hi
     B.es = c.es;
     const bool al = aligned16(W2_packed);
     hipError_t e;
-    if (mfma_stage_b(T, hidden, c.es) && mfma_down_ok(hidden, out_dim, c.M, W2_packed, W2_scale))
+    if (mfma_stage_b(T, hidden, c.es.n_pairs, c.es.n_experts) &&
+        mfma_down_ok(hidden, out_dim, c.M, W2_packed, W2_scale))
         e = mfma_down(c.M, W2_packed, W2_scale, T, hidden, out_dim, slot_tables(c.es), B.out, stream);
     else if (T == 1)
         e = al ? launch_stage_b<1, true, true, false>(B, stream)
@@ -2349,6 +2359,14 @@ extern "C" int mxfp4_moe_grouped_gemv_noalloc(const dsv4_bf16_t* x, const uint8_
     if (r != 0) return r;
     return moe_grouped_impl(x, W1_packed, W3_packed, W2_packed, W1_scale, W3_scale, W2_scale, ids, weights, T,
                             topk, n_experts, K_in, hidden, out_dim, out, ws, stream);
+}
+
+extern "C" int mxfp4_moe_decode_stages(int T, int topk, int n_experts, int K_in, int hidden, int out_dim) {
+    const int P = T * topk;
+    const bool a = mfma_stage_a(T, K_in, hidden, P, n_experts) &&
+                   mfma_swiglu_ok(K_in, hidden, nullptr, nullptr, nullptr, nullptr, nullptr);
+    const bool b = mfma_stage_b(T, hidden, P, n_experts) && mfma_down_ok(hidden, out_dim, nullptr, nullptr, nullptr);
+    return (a ? 1 : 0) | (b ? 2 : 0);
 }
 
 extern "C" int mxfp4_moe_layer(const dsv4_bf16_t* x, const float* logits,

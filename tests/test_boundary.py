@@ -256,6 +256,30 @@ def test_router_and_dispatch_validation_codes():
     assert pd(N, N, 128, 4, N, N) == -3
 
 
+# T, topk, experts, K, hidden, out_dim -> stages on the matrix cores (1: A, 2: B)
+@pytest.mark.parametrize("shape,stages", [
+    ((1, 8, 4, 4096, 2048, 4096), 0),         # one token: never
+    ((64, 8, 256, 4096, 2048, 4096), 3),
+    ((56, 8, 256, 4096, 2048, 4096), 3),      # 1.75 pairs per expert, and one token less
+    ((55, 8, 256, 4096, 2048, 4096), 0),
+    ((2, 8, 8, 4096, 2048, 4096), 1),         # 16 pairs of 2048 rows, and half the rows
+    ((2, 8, 8, 4096, 1024, 4096), 0),
+    ((2, 4, 4, 4096, 2048, 4096), 0),
+    ((4, 8, 256, 3072, 1536, 3072), 1),       # K between: 32 pairs of 1536 rows, and one row block less
+    ((4, 8, 256, 3072, 1472, 3072), 0),
+    ((2, 1, 64, 3072, 2048, 3072), 0),
+    ((64, 8, 8, 512, 2048, 4096), 2),         # K = 512 stays on the GEMV kernels
+    ((64, 8, 8, 4096, 2080, 4096), 0),        # hidden without whole row blocks or reductions
+    ((16, 2, 8, 4096, 1024, 4096), 1),        # stage B from 48 pairs
+    ((24, 2, 8, 4096, 1024, 4096), 3),
+    ((24, 2, 48, 4096, 1024, 4096), 2),
+    ((24, 2, 49, 4096, 1024, 4096), 0),
+])
+def test_decode_stage_rule(shape, stages):
+    lib = _lib("mxfp4-routed/libmxfp4_grouped_gemv.so")
+    assert lib.mxfp4_moe_decode_stages(*shape) == stages
+
+
 def test_prefill_validation_codes():
     lib = _lib("mxfp4-routed/libmxfp4_grouped_gemv.so")
     P = ctypes.c_void_p

@@ -517,27 +517,38 @@ def test_moe_scales_end_with_their_allocation(device, T):
     assert_close(host_bits(out), mx.moe_layer(x, fn, ids, w, O, n_experts=E), f"scales at the end T={T}")
 
 
-# T, topk, experts, K, hidden, out_dim, skew: every token lists expert 1 first
+def _decode_stages(*shape):
+    """Stages of a decode batch (T, topk, experts, K, hidden, out_dim) that run on
+    the matrix cores: bit 0 A, bit 1 B."""
+    return gb._load_lib().mxfp4_moe_decode_stages(*shape)
+
+
+# T, topk, experts, K, hidden, out_dim, skew (every token lists expert 1 first),
+# stages on the matrix cores (1: A, 2: B)
 DECODE_MFMA = [
-    (2, 8, 8, 1024, 256, 400, False),      # stage A only: too few pairs for stage B
-    (2, 1, 16, 3072, 256, 64, False),      # K between 2048 and 4096: stage A of any batch
-    (6, 8, 8, 1024, 256, 16, False),       # one wave per slot, eight sets of slots, one row tile
-    (13, 4, 8, 1024, 512, 48, True),       # four sets of slots
-    (17, 3, 12, 2048, 768, 400, True),     # six waves, two sets; 17 pairs on one expert
-    (12, 8, 40, 1024, 1024, 384, False),   # stage B only (fewer pairs than 1.75 per expert)
-    (33, 2, 9, 512, 1280, 3072, True),     # five waves; 16 rows per workgroup; 33 pairs
-    (64, 4, 30, 4096, 2048, 3088, True),   # eight waves, the largest batch, 193 row tiles
-    (64, 16, 3, 1024, 256, 32, True),      # duplicates in every token: 64 pairs per expert
+    (2, 8, 8, 1024, 2048, 400, False, 1),     # too few pairs for stage B
+    (2, 16, 64, 3072, 1536, 64, False, 1),    # K between 2048 and 4096: fewer pairs per expert suffice
+    (6, 8, 8, 1024, 256, 16, False, 2),       # too little work for stage A; one wave per slot, eight sets, one row tile
+    (16, 8, 8, 1024, 512, 48, True, 3),       # four sets of slots
+    (13, 4, 8, 1024, 1024, 48, True, 3),      # two sets
+    (17, 3, 12, 2048, 768, 400, True, 3),     # six waves, two sets; 17 pairs on one expert
+    (12, 8, 64, 1024, 1024, 384, False, 2),   # fewer pairs per expert than stage A takes
+    (33, 2, 9, 512, 1280, 3072, True, 2),     # K too short for stage A; five waves; 16 rows per workgroup; 33 pairs
+    (48, 2, 8, 2560, 1024, 4112, True, 3),    # 257 row tiles
+    (24, 8, 16, 2048, 2048, 2048, False, 3),  # eight waves, the most row tiles of 8
+    (64, 4, 30, 4096, 2048, 3088, True, 3),   # the largest batch, 193 row tiles
+    (64, 16, 3, 1024, 256, 32, True, 3),      # duplicates in every token: 64 pairs per expert
 ]
 
 
-@pytest.mark.parametrize("T,topk,E,K,H,O,skew", DECODE_MFMA)
-def test_decode_batches_on_matrix_cores(device, T, topk, E, K, H, O, skew):
+@pytest.mark.parametrize("T,topk,E,K,H,O,skew,stages", DECODE_MFMA)
+def test_decode_batches_on_matrix_cores(device, T, topk, E, K, H, O, skew, stages):
     """Decode batches whose stages run on the matrix cores, with ids out of
     range and duplicates, E8M0 bytes 0 and 0xFF: against the oracle and the
     general kernels (scales at an odd address), which add in another order and
     round M to bf16 from sums that differ in the last bits; bit-equal replays."""
     announce(f"decode batches on matrix cores T={T} topk={topk} E={E} K={K} H={H} O={O} skew={skew}")
+    assert _decode_stages(T, topk, E, K, H, O) == stages
     host = []
     for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
         p, s = synth.mxfp4_weight(9600 + 5 * m + T, rows, cols, E)
@@ -590,6 +601,7 @@ def test_decode_batches_largest_scales(device, big):
     give."""
     T, topk, E, K, H, O = 16, 8, 16, 1024, 512, 128
     announce(f"decode batches largest scales T={T} E={E} K={K} H={H} O={O} big={big}")
+    assert _decode_stages(T, topk, E, K, H, O) == 3
     mats = []
     for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
         p, s = synth.mxfp4_weight(9650 + 2 * m, rows, cols, E)
@@ -636,6 +648,7 @@ def test_decode_stage_a_sums_as_exact_as_general(device, K, T, E):
     over K, two above 48 tokens: 1.2 to 1.95)."""
     H, topk = 1024, 8
     announce(f"decode stage A sums K={K} T={T} E={E}")
+    assert _decode_stages(T, topk, E, K, H, H) & 1
     g = torch.Generator(device=device).manual_seed(9700 + K + T)
     nb = K // 64
     bp = torch.randperm(nb, generator=g, device=device)
@@ -678,6 +691,7 @@ def test_decode_rows_independent_of_neighbours(device):
     x = dev_bf16(synth.normal_bf16(9730, (64, K)), device)
     out = {}
     for n in (16, 32, 48, 64):
+        assert _decode_stages(n, 1, E, K, H, H) & 1
         ids = torch.full((n, 1), 2, dtype=torch.int32, device=device)
         out[n] = gb.mxfp4_moe_grouped_gemv(x[:n].contiguous(), *mats, ids, torch.ones((n, 1), device=device))
     for n in (16, 32, 48):
@@ -688,6 +702,7 @@ def test_decode_overflow_stays_infinite(device):
     """Sums beyond fp32 give the infinities of the general kernels, no NaN."""
     T, E, K, H, O = 24, 2, 1024, 2048, 64
     announce(f"decode overflow T={T} K={K} H={H}")
+    assert _decode_stages(T, 1, E, K, H, O) & 1
     g = torch.Generator(device=device).manual_seed(9740)
 
     def positive(rows, cols, byte):
@@ -712,6 +727,7 @@ def test_decode_stage_b_adds_waves_in_double(device):
     them have to give the 1, which fp32 sums in wave order lose."""
     T, E, K, H, O = 64, 2, 2048, 2048, 4096
     announce(f"decode stage B sums of the waves T={T} H={H} O={O}")
+    assert _decode_stages(T, 1, E, K, H, O) & 2
     W1 = np.zeros((E, H, K // 2), np.uint8)
     W1[..., 0] = 0x02                              # W1 x = x[0] = 128, and so is its silu
     W2 = np.zeros((E, O, H // 2), np.uint8)
@@ -738,6 +754,7 @@ def test_decode_batches_smallest_scales(device, small, K, H):
     sums and M. One expert of W2 has no such byte."""
     T, topk, E, O = 33, 8, 16, 192
     announce(f"decode batches smallest scales K={K} H={H} matrix {small}")
+    assert _decode_stages(T, topk, E, K, H, O) == 3
     rng = np.random.default_rng(9750 + K)
     mats = []
     for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
