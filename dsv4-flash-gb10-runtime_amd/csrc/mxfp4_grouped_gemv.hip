@@ -1902,11 +1902,19 @@ int launch_route(const float* logits, const int32_t* ids, const float* weights, 
 //     17.4 / 17.0, 16 26.3 / 28.8, 32 47.9 / 53.8, P / E = 1 227 / 308; 2560 (hidden
 //     1536) 16 pairs 21.3 / 19.5, 24 30.7 / 27.2, 32 32.7 / 32.9, 64 58.6 / 61.0,
 //     P / E = 1 144 / 197; 3584 (1408) 24 38.8 / 35.0, 32 40.6 / 44.3.
-//   B, hidden = 2048: 1 204 / 214, 1.5 274 / 272 and 148 / 149, 1.75 161 / 157,
-//     2 181 / 175, 338 / 320, 663 / 627; hidden = 1536: 0.75 145.6 / 146.4, 1.12
-//     193 / 183 and 369 / 349; 1024: 0.5 98 / 89 and 34 / 37, 1 53.2 / 52.6 and
-//     165 / 143. Few pairs leave too few slots for its ring: 16 pairs 38 / 42, 32
-//     61.9 / 62.0, 31.7 / 32.0 and 38 / 41, 48 71 / 64, 64 99 / 96.
+//   B: the MFMA kernel takes about the same time for any out_dim up to 2048 and
+//     from there to 4096 (one round of workgroups of 8 or 16 rows), the GEMV
+//     kernels another round for every 2048 rows; where they take an odd number
+//     of rounds, the MFMA kernel's last is half empty. hidden = 2048, P / E =
+//     1.75: out_dim = 4096 209 / 235 and 58 / 65, 2560 56 / 58, 8192 404 / 435;
+//     2048 51 / 39, at 3 59 / 58, at 3.5 61 / 65; 6144 106 / 90, 5120 at 2.75
+//     118 / 118, at 3 123 / 127. hidden = 1536 (1280 and 1792 likewise): 4096 at 1
+//     34.3 / 34.1 (48 pairs), 41.9 / 42.5 (64) and 137 / 149 (256); 2048 at 2 50 / 47, at 2.5
+//     53 / 54; 6144 at 2 101 / 92, at 2.5 105 / 109. hidden <= 1024: at 1 25 / 28
+//     (2048), 27 / 39 (4096), 50.4 / 50.9 and 41.3 / 39.9 (5120). Few slots leave
+//     its ring unfilled: at out_dim = 4096 16 pairs 38 / 42, 32 61.9 / 62.0 and
+//     31.7 / 32.0 (GEMV / MFMA), 48 64 / 71; at out_dim = 2048, hidden = 2048 8
+//     tokens x 8 of 8 experts 19.3 / 17.6, 16 x 4 of 16 22.0 / 23.4.
 bool mfma_stage_a(int T, int K, int hidden, int n_pairs, int n_experts) {
     const int work = n_pairs * hidden;            // at most 1024 * 4096
     if (T < 2) return false;
@@ -1914,9 +1922,21 @@ bool mfma_stage_a(int T, int K, int hidden, int n_pairs, int n_experts) {
     return K > 2048 && K < 4096 && work >= 32 * 1536;
 }
 
-bool mfma_stage_b(int T, int hidden, int n_pairs, int n_experts) {
-    return T > 1 && n_pairs >= 48 &&
-           (hidden < 2048 ? n_pairs >= n_experts : 4 * n_pairs >= 7 * n_experts);
+bool mfma_stage_b(int T, int hidden, int out_dim, int n_pairs, int n_experts) {
+    if (T < 2 || n_pairs < 48) return false;
+    const int rounds = (out_dim + 2047) / 2048;   // of the GEMV kernels: 8 rows on each of 256 CUs
+    int quarters;                                 // least pairs per expert, times 4
+    if (hidden <= 1024) {
+        quarters = rounds == 3 ? 5 : 4;
+    } else if (rounds == 1) {
+        if (T < 16) return false;
+        quarters = hidden < 2048 ? 10 : 14;
+    } else if (rounds % 2 != 0) {
+        quarters = hidden < 2048 ? 10 : 11;
+    } else {
+        quarters = hidden < 2048 ? (n_pairs < 128 ? 5 : 4) : 7;
+    }
+    return 4 * n_pairs >= quarters * n_experts;
 }
 
 SlotTables slot_tables(const ExpertSet& es) {
@@ -1974,7 +1994,7 @@ int launch_down(const uint8_t* W2_packed, const uint8_t* W2_scale, int T, int hi
     B.es = c.es;
     const bool al = aligned16(W2_packed);
     hipError_t e;
-    if (mfma_stage_b(T, hidden, c.es.n_pairs, c.es.n_experts) &&
+    if (mfma_stage_b(T, hidden, out_dim, c.es.n_pairs, c.es.n_experts) &&
         mfma_down_ok(hidden, out_dim, c.M, W2_packed, W2_scale))
         e = mfma_down(c.M, W2_packed, W2_scale, T, hidden, out_dim, slot_tables(c.es), B.out, stream);
     else if (T == 1)
@@ -2365,7 +2385,8 @@ extern "C" int mxfp4_moe_decode_stages(int T, int topk, int n_experts, int K_in,
     const int P = T * topk;
     const bool a = mfma_stage_a(T, K_in, hidden, P, n_experts) &&
                    mfma_swiglu_ok(K_in, hidden, nullptr, nullptr, nullptr, nullptr, nullptr);
-    const bool b = mfma_stage_b(T, hidden, P, n_experts) && mfma_down_ok(hidden, out_dim, nullptr, nullptr, nullptr);
+    const bool b = mfma_stage_b(T, hidden, out_dim, P, n_experts) &&
+                   mfma_down_ok(hidden, out_dim, nullptr, nullptr, nullptr);
     return (a ? 1 : 0) | (b ? 2 : 0);
 }
 

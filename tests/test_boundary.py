@@ -274,6 +274,20 @@ def test_router_and_dispatch_validation_codes():
     ((24, 2, 8, 4096, 1024, 4096), 3),
     ((24, 2, 48, 4096, 1024, 4096), 2),
     ((24, 2, 49, 4096, 1024, 4096), 0),
+    ((64, 8, 256, 4096, 2048, 2048), 1),      # one round of 8 rows: 3.5 pairs per expert at hidden = 2048
+    ((28, 8, 64, 4096, 2048, 2048), 3),
+    ((64, 8, 256, 4096, 2048, 2056), 1),      # out_dim without whole row tiles
+    ((64, 8, 256, 4096, 2048, 2064), 3),      # two rounds
+    ((64, 8, 256, 4096, 2048, 5120), 1),      # three
+    ((22, 8, 64, 4096, 2048, 5120), 3),
+    ((15, 8, 120, 2048, 1536, 4096), 0),      # hidden = 1536: 1.25 pairs per expert, 1 from 128 pairs
+    ((15, 8, 96, 2048, 1536, 4096), 2),
+    ((16, 8, 128, 2048, 1536, 4096), 2),
+    ((32, 8, 128, 2048, 1536, 2048), 1),      # 2.5 in one round
+    ((40, 8, 128, 2048, 1536, 2048), 3),
+    ((8, 8, 8, 4096, 2048, 2048), 1),         # few tokens in one round
+    ((32, 8, 256, 2048, 1024, 6144), 0),      # 1.25 in three rounds at hidden = 1024
+    ((40, 8, 256, 2048, 1024, 6144), 2),
 ])
 def test_decode_stage_rule(shape, stages):
     lib = _lib("mxfp4-routed/libmxfp4_grouped_gemv.so")
