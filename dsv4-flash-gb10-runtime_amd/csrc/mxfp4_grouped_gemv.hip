@@ -1849,16 +1849,19 @@ MoeCall moe_call(int T, int topk, int n_experts, int hidden, void* workspace) {
     return c;
 }
 
-// Up to this many tokens the routing kernel ranks the logits itself (16 waves,
-// one token each); for more, one-wave workgroups rank them first, in a launch
-// of their own (top-8 of 256 at T = 40: 17 us in one launch, 6 + 5 in two; at
-// T = 16 6.4 against 2.6 + 2.6 and the second launch).
-constexpr int kRouteRankTok = 16;
+// Whether the logits of a batch are ranked by one-wave workgroups in a launch of
+// their own; the routing kernel ranks them itself otherwise (16 waves, one token
+// each at a time). Layers of 256 experts (sigmoid; us, own launch / not): T = 17
+// 29.2 / 28.6 (top-1), 74.6 / 74.5 (top-4), 20 31.8 / 31.3 (top-1), 24 36.1 /
+// 35.9 and 145.4 / 146.1 (top-8 of 64), 32 43.7 / 44.3, 117 / 119 (top-4) and 183 /
+// 186 (top-8), 64 69.5 / 72.5; the square root scores cost more: top-2 at 17 50.9 /
+// 52.6, top-6 at 17 107 / 109, at 32 165 / 173.
+bool rank_apart(int T, const Scoring& sc) { return T > (sc.mode == kScoreSigmoid ? 20 : 16); }
 
 int launch_route(const float* logits, const int32_t* ids, const float* weights, int T, int topk,
                  int n_experts, int32_t* ids_out, float* w_out, const MoeCall& c,
                  hipStream_t stream, Scoring sc = Scoring{kScoreSigmoid, 1.0f}) {
-    if (logits != nullptr && T > kRouteRankTok) {
+    if (logits != nullptr && rank_apart(T, sc)) {
         // The picks pass through the caller's outputs, or through the pair
         // tables, which the routing kernel reads in full before it writes them.
         int32_t* picks = ids_out != nullptr ? ids_out : c.rt.pair_tok;

@@ -466,9 +466,9 @@ def test_router_logits_token_groups(device, K):
 
 
 @pytest.mark.parametrize("outputs", ["both", "none", "ids", "weights"])
-@pytest.mark.parametrize("T", [16, 17, 64])
+@pytest.mark.parametrize("T", [16, 17, 20, 21, 64])
 def test_layer_gating_of_larger_batches(device, T, outputs):
-    """Above 16 tokens the logits are ranked in a launch of its own, whose picks
+    """Above 20 tokens the logits are ranked in a launch of its own, whose picks
     pass through the requested outputs or through the pair tables: the layer has
     to equal the layer on the caller's routing, bit for bit."""
     E, K, H, O, topk = 40, 512, 256, 128, 8
@@ -483,6 +483,29 @@ def test_layer_gating_of_larger_batches(device, T, outputs):
     io = torch.full_like(ids, -7) if outputs in ("both", "ids") else None
     wo = torch.full_like(w, -7.0) if outputs in ("both", "weights") else None
     got = gb.mxfp4_moe_layer(x, logits, W1, W3, W2, topk, ids_out=io, weights_out=wo)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert io is None or torch.equal(io, ids)
+    assert wo is None or torch.equal(wo, w)
+
+
+@pytest.mark.parametrize("outputs", ["both", "none", "ids", "weights"])
+@pytest.mark.parametrize("T", [16, 17, 64])
+def test_dispatch_gating_of_larger_batches(device, T, outputs):
+    """The routed dispatch ranks the square-root scores in a launch of its own
+    above 16 tokens: it has to equal the layer on the routing of
+    router_logits + route_topk, bit for bit."""
+    E, K, H, O, topk = 200, 512, 256, 128, 6
+    announce(f"mxfp4_moe_routed_dispatch gating T={T} outputs={outputs}")
+    W1, W3, W2 = ({"packed": dev_u8(p, device), "scale": dev_u8(s, device)}
+                  for p, s in (synth.mxfp4_weight(9420 + 2 * m, r, c, E)
+                               for m, (r, c) in enumerate(((H, K), (H, K), (O, H)))))
+    x = dev_bf16(synth.normal_bf16(9430, (T, K)), device)
+    wg = dev_bf16(synth.normal_bf16(9431 + T, (E, K), 0.05), device)
+    ids, w = gb.route_topk(gb.router_logits(x, wg), topk, gb.SCORE_SQRT_SOFTPLUS, 1.5)
+    want = gb.mxfp4_moe_grouped_gemv(x, W1, W3, W2, ids, w)
+    io = torch.full_like(ids, -7) if outputs in ("both", "ids") else None
+    wo = torch.full_like(w, -7.0) if outputs in ("both", "weights") else None
+    got = gb.mxfp4_moe_routed_dispatch(x, wg, W1, W3, W2, topk, ids_out=io, weights_out=wo)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     assert io is None or torch.equal(io, ids)
     assert wo is None or torch.equal(wo, w)
