@@ -42,3 +42,7 @@ hipError_t mfma_down(const uint16_t* M, const uint8_t* w2, const uint8_t* s2, in
 // matrix cores: bit 0 stage A, bit 1 stage B (so that the tests can name the
 // path that a case takes; needs no GPU).
 extern "C" int mxfp4_moe_decode_stages(int T, int topk, int n_experts, int K_in, int hidden, int out_dim);
+
+// Whether a prefill chunk with 16-byte aligned scales takes the wide tiles
+// (likewise).
+extern "C" int mxfp4_moe_prefill_wide(int T, int topk, int n_experts, int K_in, int hidden, int out_dim);

@@ -294,6 +294,31 @@ def test_decode_stage_rule(shape, stages):
     assert lib.mxfp4_moe_decode_stages(*shape) == stages
 
 
+@pytest.mark.parametrize("shape,wide", [
+    ((512, 8, 256, 4096, 2048, 4096), 1),
+    ((384, 8, 256, 4096, 2048, 4096), 1),     # 12 pairs per expert, and one token less
+    ((383, 8, 256, 4096, 2048, 4096), 0),
+    ((16384, 16, 256, 8192, 8192, 8192), 1),  # the largest: no overflow
+    ((1024, 1, 4, 4096, 2048, 4096), 1),      # pairs x rows, one pair less, few experts
+    ((1023, 1, 4, 4096, 2048, 4096), 0),
+    ((1024, 1, 2, 4096, 2048, 4096), 0),
+    ((1280, 1, 2, 4096, 2048, 4096), 1),
+    ((2047, 1, 8, 2048, 1024, 2048), 0),
+    ((2048, 1, 8, 2048, 1024, 2048), 1),
+    ((4096, 1, 8, 4096, 512, 4096), 1),       # stage A's rows, stage B's
+    ((4095, 1, 8, 4096, 512, 4096), 0),
+    ((4096, 1, 8, 512, 4096, 512), 0),
+    ((8192, 1, 8, 512, 4096, 512), 1),
+    ((1024, 1, 8, 4096, 2048, 256), 1),       # a short stage B does not count
+    ((768, 1, 16, 4096, 2048, 4096), 1),      # 24 pairs each of many experts
+    ((383, 1, 16, 4096, 2048, 4096), 0),
+    ((384, 1, 15, 4096, 2048, 4096), 0),
+])
+def test_prefill_tile_rule(shape, wide):
+    lib = _lib("mxfp4-routed/libmxfp4_grouped_gemv.so")
+    assert lib.mxfp4_moe_prefill_wide(*shape) == wide
+
+
 def test_prefill_validation_codes():
     lib = _lib("mxfp4-routed/libmxfp4_grouped_gemv.so")
     P = ctypes.c_void_p

@@ -378,14 +378,15 @@ def _pairs_with_counts(counts, topk, seed):
 
 
 @pytest.mark.parametrize("K,H,O,counts,topk", [
-    (512, 512, 64, _TILE_EDGES, 2),                # every tile size; one macro-step pair, a quarter-full row block
-    (1536, 512, 320, _TILE_EDGES[::2], 3),         # 3 x 512: the four-deep weight ring ends mid-way
-    (512, 1536, 576, _TILE_EDGES[1::3], 1),
-    (4096, 512, 256, [1, 16, 40, 64, 100, 128], 2),
-    (512, 8192, 192, [20, 60, 120, 130], 2),
+    (512, 2048, 64, _TILE_EDGES, 2),               # every tile size; one macro-step pair in stage A, a quarter-full row block
+    (1536, 2560, 320, _TILE_EDGES[::2], 3),        # 3 and 5 x 512: the four-deep weight ring ends mid-way
+    (2560, 3072, 576, _TILE_EDGES[1::2], 1),
+    (4096, 2048, 256, [1, 16, 40, 64, 100, 128, 900], 2),
+    (1024, 8192, 192, [20, 60, 120, 130], 2),
+    (1024, 512, 1024, [3, 70, 1100, 129, 2900], 2),  # one macro-step pair in stage B
 ])
 def test_prefill_wide_tiles_equal_small_tiles(device, K, H, O, counts, topk):
-    """Chunks with 12 or more pairs per expert run on the wide tiles. The same
+    """Chunks of many pairs, 12 or more per expert, run on the wide tiles. The same
     chunk with more (unrouted) experts in the tensors runs on the 64 x 64 tiles:
     same weights, k order, sums and rounding, so the same bits. Special scale
     bytes (0xFF and 0) are among the blocks."""
@@ -394,7 +395,8 @@ def test_prefill_wide_tiles_equal_small_tiles(device, K, H, O, counts, topk):
     T = ids.shape[0]
     E_all = T * topk // 12 + 1
     announce(f"mxfp4_moe_prefill wide tiles K={K} H={H} O={O} T={T} topk={topk} E={E} / {E_all}")
-    assert T * topk >= 12 * E and T * topk < 12 * E_all and E_all >= E
+    wide_rule = gb._load_lib().mxfp4_moe_prefill_wide
+    assert wide_rule(T, topk, E, K, H, O) and not wide_rule(T, topk, E_all, K, H, O) and E_all >= E
     rng = np.random.default_rng(9001 + K)
     mats = []
     for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
@@ -416,7 +418,7 @@ def test_prefill_wide_tiles_equal_small_tiles(device, K, H, O, counts, topk):
     # scale rows that are not 16-byte aligned keep the 64 x 64 tiles
     off = [{"packed": d["packed"], "scale": _at_offset(d["scale"], 4)} for d in few]
     assert np.array_equal(host_bits(gb.mxfp4_moe_prefill(xd, *off, idd, wd)), wide)
-    if K * H <= 512 * 512:
+    if K == 512:
         def fn(e):
             return tuple((p[e], s[e]) for p, s, _ in mats)
 
