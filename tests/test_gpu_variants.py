@@ -451,6 +451,28 @@ def test_prefill_routing_of_large_chunks(device, T, topk, E):
         assert torch.equal(part.view(torch.int16), whole[t0:t0 + 512].view(torch.int16)), t0
 
 
+@pytest.mark.parametrize("topk", [1, 2, 3, 4, 5, 8, 9, 16])
+def test_prefill_combine_of_every_topk(device, topk):
+    """The combine keeps 1, 2, 4 or 8 rows in flight: against the oracle, with ids
+    out of range (a token without any among them) and duplicates."""
+    T, E, K, H, O = 19, 8, 512, 512, 1088
+    announce(f"mxfp4_moe_prefill combine topk={topk} T={T} O={O}")
+    host = [synth.mxfp4_weight(9120 + 2 * m, rows, cols, E) for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H)))]
+    rng = np.random.default_rng(9130 + topk)
+    ids = rng.integers(-1, E + 1, (T, topk)).astype(np.int32)
+    ids[3], ids[7] = -1, 5
+    w = (rng.random((T, topk)) + 0.1).astype(np.float32)
+    x = synth.normal_bf16(9131, (T, K))
+    mats = [{"packed": dev_u8(p, device), "scale": dev_u8(s, device)} for p, s in host]
+    out = host_bits(gb.mxfp4_moe_prefill(dev_bf16(x, device), *mats, torch.from_numpy(ids).to(device), dev_f32(w, device)))
+    assert not out[3].any()
+
+    def fn(e):
+        return tuple((p[e], s[e]) for p, s in host)
+
+    assert_close(out, mx.moe_layer(x, fn, ids, w, O, n_experts=E), f"combine topk={topk}")
+
+
 # ------------------------------------------------- routing of larger batches ---
 
 @pytest.mark.parametrize("K", [1000, 4096])
