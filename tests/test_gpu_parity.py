@@ -542,9 +542,9 @@ def test_moe_one_token_ids_path(device, ids_row, K):
                                        (2048, "ragged")])
 def test_moe_multi_token_many_pairs_per_expert(device, K, routing):
     """Several tokens on the aligned path (K = 2048 or 4096, hidden = 2048) with
-    16 experts, so each expert serves many tokens: the multi-token stage A
-    stages the pairs after the first in passes, and the multi-token stage B
-    loads their M slices on demand. "shared": every token routes to the same
+    16 experts, so each expert serves many tokens and both stages run on the
+    matrix cores (the GEMV kernels with many pairs per expert:
+    test_moe_multi_token_gemv_hot_experts). "shared": every token routes to the same
     8 experts (16 pairs each); "ragged": 1 to 16 pairs per expert."""
     E, H, O, T, topk = 16, 2048, 256, 16, 8
     announce(f"mxfp4_moe_grouped_gemv T={T} E={E} K={K} routing={routing}")
@@ -574,6 +574,42 @@ def test_moe_multi_token_many_pairs_per_expert(device, K, routing):
         return (W1p[e], W1s[e]), (W3p[e], W3s[e]), (W2p[e], W2s[e])
 
     assert_close(host_bits(out), mx.moe_layer(x, fn, ids, w, O), f"moe T={T} K={K} {routing}")
+
+
+@pytest.mark.parametrize("T,topk,E", [(2, 4, 16), (16, 8, 80), (17, 6, 64), (40, 4, 96), (64, 2, 80)])
+@pytest.mark.parametrize("K", [2048, 4096])
+def test_moe_multi_token_gemv_hot_experts(device, K, T, topk, E):
+    """Batches whose experts are many enough for the multi-token GEMV kernels
+    (hidden = 2048) while every token goes to a few of them, from one to all: the
+    further-pair passes of stage A, the M slices that stage B loads on demand and
+    its bodies for up to 16 and up to 64 tokens."""
+    H, O = 2048, 200
+    announce(f"mxfp4_moe_grouped_gemv hot experts T={T} topk={topk} E={E} K={K}")
+    assert gb._load_lib().mxfp4_moe_decode_stages(T, topk, E, K, H, O) == 0
+    rng = np.random.default_rng(8540 + T)
+    hot = np.sort(rng.choice(E, topk + 2, replace=False)).astype(np.int32)
+    host, mats = [], []
+    for m, (rows, cols) in enumerate(((H, K), (H, K), (O, H))):
+        p, s = synth.mxfp4_weight(8550 + 2 * m, rows, cols, len(hot))
+        host.append((p, s))
+        pd = torch.zeros((E, rows, cols // 2), dtype=torch.uint8, device=device)
+        sd = torch.zeros((E, rows, cols // 32), dtype=torch.uint8, device=device)
+        pd[hot], sd[hot] = dev_u8(p, device), dev_u8(s, device)
+        mats.append({"packed": pd, "scale": sd})
+    # hot expert 0 of every token, the others of a falling share of them
+    ids = np.empty((T, topk), np.int32)
+    for t in range(T):
+        rest = 1 + rng.choice(topk + 1, topk - 1, replace=False, p=np.arange(topk + 1, 0, -1) / ((topk + 1) * (topk + 2) / 2))
+        ids[t] = hot[np.concatenate([[0], rest])]
+    w = (rng.random((T, topk)) + 0.1).astype(np.float32)
+    x = synth.normal_bf16(8560 + K, (T, K))
+    out = gb.mxfp4_moe_grouped_gemv(dev_bf16(x, device), *mats, torch.from_numpy(ids).to(device), dev_f32(w, device))
+    where = {int(e): i for i, e in enumerate(hot)}
+
+    def fn(e):
+        return tuple((p[where[e]], s[where[e]]) for p, s in host)
+
+    assert_close(host_bits(out), mx.moe_layer(x, fn, ids, w, O, n_experts=E), f"hot experts T={T} K={K}")
 
 
 @pytest.mark.parametrize("T", [1, 4])
