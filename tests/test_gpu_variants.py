@@ -816,6 +816,7 @@ def test_decode_batches_smallest_scales(device, small, K, H):
     scale = 1.0 if small == 2 else 2.0 ** 100      # the other of W1 x and W3 x about 2^100
     x = mx.bf16_round(mx.bf16_to_f32(synth.normal_bf16(9770, (T, K))) * np.float32(scale))
     ids = np.stack([rng.permutation(E)[:topk] for _ in range(T)]).astype(np.int32)
+    ids[:, 0] = 1                                  # 33 pairs on one expert
     w = (rng.random((T, topk)) + 0.1).astype(np.float32)
     args = torch.from_numpy(ids).to(device), dev_f32(w, device)
     gen = [{"packed": m["packed"], "scale": _at_offset(m["scale"], 1)} for m in mats]
