@@ -120,7 +120,10 @@ size_t mxfp4_moe_workspace_bytes(int T, int topk, int n_experts, int hidden);
  * Expert-indexed multi-token routed SwiGLU MoE: experts are read in place from
  * per-layer tensors W1/W3 [n_experts, hidden, K_in/2], W2 [n_experts, out_dim,
  * hidden/2] (+ scales), each unique routed expert is streamed once for all of
- * its tokens; one launch per projection (stage A: W1+W3, stage B: W2).
+ * its tokens; one launch per projection (stage A: W1+W3, stage B: W2). Batches
+ * with about two or more tokens per expert run on the matrix cores, the others
+ * on the vector units: the sums are fp32 in both (stage B's last in fp64 on the
+ * matrix cores) and differ in order.
  *   out[t] = bf16( sum_k weights[t,k] * W2_{ids[t,k]} . bf16(silu(W1 x_t) * (W3 x_t)) )
  * x [T, K_in] bf16, ids/weights [T, topk], out [T, out_dim] bf16.
  * Returns 0; -1 K_in%32; -2 hidden%32; -3 K_in/hidden > 4096; -4 bad
@@ -185,8 +188,9 @@ int mxfp4_moe_down(const uint8_t* W2_packed, const uint8_t* W2_scale, int T, int
                    int n_experts, int hidden, int out_dim, dsv4_bf16_t* out, void* workspace,
                    hipStream_t stream);
 
-/* EXTENSION: one routed-MoE layer at decode in one call (three launches on
- * `stream`): device gating of logits [T, n_experts] (top-`topk`, sigmoid
+/* EXTENSION: one routed-MoE layer at decode in one call (two launches on
+ * `stream` for one token on the aligned path, three otherwise, four above 20
+ * tokens): device gating of logits [T, n_experts] (top-`topk`, sigmoid
  * weights renormalised to 1, as mxfp4_moe_route_sigmoid_topk), then stages A
  * and B of mxfp4_moe_grouped_gemv. ids_out / weights_out ([T, topk]; either
  * or both may be NULL) receive the routing. Workspace as mxfp4_moe_grouped_gemv. Return codes
@@ -199,10 +203,10 @@ int mxfp4_moe_layer(const dsv4_bf16_t* x, const float* logits,
                     hipStream_t stream);
 
 /* EXTENSION: the first part of mxfp4_moe_layer (gating of logits and stage A,
- * one launch for one token on the aligned path, two otherwise); followed by
- * mxfp4_moe_down with the same workspace it completes the layer with the same
- * bits. For callers that schedule the projections themselves and for
- * per-launch timing. Arguments and return codes as mxfp4_moe_layer. */
+ * one launch for one token on the aligned path, two otherwise, three above 20
+ * tokens); followed by mxfp4_moe_down with the same workspace it completes the
+ * layer with the same bits. For callers that schedule the projections
+ * themselves and for per-launch timing. Arguments and return codes as mxfp4_moe_layer. */
 int mxfp4_moe_gate_swiglu(const dsv4_bf16_t* x, const float* logits, const uint8_t* W1_packed,
                           const uint8_t* W3_packed, const uint8_t* W1_scale, const uint8_t* W3_scale,
                           int T, int topk, int n_experts, int K_in, int hidden, int32_t* ids_out,
@@ -215,8 +219,8 @@ int mxfp4_moe_gate_swiglu(const dsv4_bf16_t* x, const float* logits, const uint8
  * 1.5 in the reference) and stages A and B of mxfp4_moe_grouped_gemv, with the
  * experts read in place from the per-layer tensors. No host sync, no pack
  * copies; three launches for one token (the scoring runs inside stage A), four
- * otherwise. W_gate [n_experts, K_in] bf16; ids_out / weights_out as
- * mxfp4_moe_layer. Workspace of mxfp4_moe_dispatch_workspace_bytes bytes.
+ * for up to 16, five for more. W_gate [n_experts, K_in] bf16; ids_out /
+ * weights_out as mxfp4_moe_layer. Workspace of mxfp4_moe_dispatch_workspace_bytes bytes.
  * Returns as mxfp4_moe_layer, plus -3 for an unaligned x or W_gate and -4 for
  * T, n_experts or K_in outside the router's limits. */
 size_t mxfp4_moe_dispatch_workspace_bytes(int T, int topk, int n_experts, int hidden);
@@ -235,8 +239,9 @@ int mxfp4_moe_routed_dispatch(const dsv4_bf16_t* x, const dsv4_bf16_t* W_gate,
  * with the MXFP4 weights dequantised exactly to bf16 and multiplied on
  * v_mfma_f32_16x16x32_bf16 (fp32 accumulate). x [T, K_in] bf16 (16-byte
  * aligned), ids/weights [T, topk], out [T, out_dim] bf16. Ids outside
- * [0, n_experts) contribute nothing. Four launches, no allocation; workspace
- * of mxfp4_moe_prefill_workspace_bytes bytes (0 for invalid arguments).
+ * [0, n_experts) contribute nothing. Four launches (five above 8192 entries
+ * T * topk), no allocation; workspace of mxfp4_moe_prefill_workspace_bytes
+ * bytes (0 for invalid arguments).
  * Returns 0; -1 K_in not a multiple of 512 in [512, 8192]; -2 hidden likewise;
  * -3 out_dim not a positive multiple of 64, a null or unaligned operand; -4 T outside
  * [1, 16384], topk outside [1, 16] or n_experts outside [1, 1024]; -5..-8
